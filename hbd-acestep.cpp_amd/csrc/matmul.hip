@@ -589,6 +589,7 @@ typedef int mm_i32x4 __attribute__((ext_vector_type(4)));
 typedef int mm_i32x16 __attribute__((ext_vector_type(16)));
 typedef float mm_f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 mm_f16x8 __attribute__((ext_vector_type(8)));
+typedef float mm_f32x32 __attribute__((ext_vector_type(32)));
 
 __global__ void __launch_bounds__(256) k_mmq_q8_0(const MmvArgs a) {
     const int      tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
@@ -749,6 +750,295 @@ __global__ void __launch_bounds__(256) k_mmq_q8_0(const MmvArgs a) {
     }
 }
 
+// Matrix kernel for grids that the 128 x 128 tiles leave idle (short x: short
+// prompts and clips, a few rows more than the matrix-vector kernel takes): a
+// workgroup owns 64 rows of x x 64 weight rows, and its 8 waves are 2 positions (32
+// rows of x x 64 weight rows each) x 4 key groups: every stage of 4 blocks gives each
+// key group one, and the groups' sums are added in group order in LDS, so the keys
+// are split over 4 waves without partials in memory or a second launch. What bounds
+// it is the latency of one wave's chain of blocks (an LDS read, two MFMAs, 64
+// conversions and fmas), so the split is over keys and the operands are fetched ahead:
+// global_load_lds copies them into LDS 3 stages (12 blocks) before use, in MFMA lane
+// order, so that the reads are linear and conflict-free; up to 128 VGPRs keep 4 waves
+// per SIMD (2 workgroups per CU). The block's scales are two f32 outer products by one
+// v_mfma_f32_32x32x1_2b (K = 1: a lane holds one d_x and one d_w, no zero slots to
+// build). Measured against the 128 x 128 kernel (x quantization and split sum
+// included, us, 2048 -> 2048 / 2048 -> 12288): 9 rows 27.5 ->
+// 13.2 / 30.2 -> 16.7, 128 rows 28.4 -> 14.5 / 35.2 -> 23.4, 375 rows 32.7 -> 17.8 /
+// 54.8 -> 49.3, 1537 rows of 2048 -> 2048 45.9 -> 42.9. On large grids it loses
+// (12288 x 1024 rows: 110 against 89): twice the operand traffic per output.
+
+// 16 bytes per lane from base + off straight into LDS at dst + 16 * lane (dst uniform)
+__device__ __forceinline__ void mmq_dma(uint32_t dst, const char * base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(dst), "v"(off), "s"(base)
+                 : "memory", "m0");
+}
+__device__ __forceinline__ void mmq_dma_v(uint32_t dst, const char * p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :
+                 : "s"(dst), "v"(p)
+                 : "memory", "m0");
+}
+
+__global__ void __launch_bounds__(512, 4) k_mmq64_q8_0(const MmvArgs a) {
+    // 32-row tiles per wave (of x, of w), wave positions, key groups, blocks per stage, stages
+    constexpr int WM = 1, WN = 2, NM = 2, NN = 1, KG = 4, KB = 4, D = 4;
+    static_assert(WN % 2 == 0 && KB % KG == 0, "the scales of two weight tiles come from one MFMA");
+    constexpr int XT = WM * NM, WT = WN * NN, NP = NM * NN, NW = NP * KG;  // 32-row tiles, wave positions, waves
+    constexpr int QI    = KB * (XT + WT);                                   // 1 KB loads of a stage's quants
+    constexpr int XS    = KB * XT * 8, WS = KB * WT * 4;                    // 16-byte chunks of its scales of x, of w
+    constexpr int SCI   = (XS + WS + 63) / 64;                              // 1 KB loads of those
+    constexpr int STAGE = QI * 1024 + (XS + WS) * 16;
+    constexpr int RED   = NW * WM * WN * 4096;                              // the key groups' sums
+    static_assert(QI % NW == 0 && SCI <= NW, "every wave issues QI / NW loads, the first SCI waves one more");
+    __shared__ __attribute__((aligned(1024))) char lds[D * STAGE > RED ? D * STAGE : RED];
+    const int      tid = threadIdx.x, l = tid & 63;
+    const int      wv  = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int      hh  = l >> 5, c = l & 31;
+    // Workgroups go to the XCDs in turn: each XCD takes one run of tiles, in
+    // groups of 8 row tiles, so that the tiles resident on it share x and w in its L2.
+    const uint32_t tn = (a.n + 32 * WT - 1) / (32 * WT), tm = (a.m + 32 * XT - 1) / (32 * XT);
+    const uint32_t per = tn * tm, total = per * a.splits;
+    uint32_t       t   = blockIdx.x;
+    {
+        const uint32_t x8 = t % 8, q = total / 8, r = total % 8;
+        t = x8 * q + (x8 < r ? x8 : r) + t / 8;
+    }
+    const uint32_t z = t / per;
+    t -= z * per;
+    const uint32_t gm = t / (8 * tn), gh = tm - 8 * gm < 8 ? tm - 8 * gm : 8;
+    t -= gm * 8 * tn;
+    const uint32_t nt = t / gh, mt = 8 * gm + (t - nt * gh);
+    const uint32_t mw = mt * 32 * XT, nw = nt * 32 * WT;  // the workgroup's first rows of x and of w
+    // this workgroup's blocks: split z of the key range
+    const uint32_t bb = z * a.bps;
+    const uint32_t be = bb + a.bps < a.nbk ? bb + a.bps : a.nbk;
+
+    const uint32_t lds0  = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) lds;
+    const uint64_t xqs   = (uint64_t) a.mp * 32;  // quants of x per block
+    const uint32_t xoff  = (uint32_t) (c * 32 + hh * 16), woff = (uint32_t) (hh * 1024 + c * 16);
+    // A stage's loads: every 1 KB tile lands in LDS in MFMA lane order (lane l: row
+    // l % 32, bytes 16 (l / 32) of the block), so the reads are linear; blocks past
+    // the split's end and row groups past the weight are clamped (never used / stored).
+    auto issue = [&](uint32_t b, uint32_t buf) {
+        const uint32_t base = lds0 + buf * STAGE;
+#pragma unroll
+        for (int i = 0; i < QI / NW; ++i) {
+            const int      o = wv + NW * i, kb = o / (XT + WT), r = o % (XT + WT);
+            const uint32_t bk = b + kb < a.nbk ? b + kb : a.nbk - 1;
+            if (r < XT) {
+                mmq_dma(base + (uint32_t) o * 1024, a.xq + bk * xqs + (uint64_t) (mw + 32 * r) * 32, xoff);
+            } else {
+                const uint32_t g0 = nw / 64 + (r - XT) / 2, g = g0 < a.ng ? g0 : a.ng - 1;
+                mmq_dma(base + (uint32_t) o * 1024, a.w + ((uint64_t) g * a.nbk + bk) * 2048 + 512 * ((r - XT) & 1), woff);
+            }
+        }
+        if (wv < SCI) {
+            const uint32_t q = (uint32_t) (wv * 64 + l);  // 16-byte chunk: x scales [kb][32 XT] f32, then w's [kb][32 WT] fp16
+            const char *   p = nullptr;
+            if (q < XS) {
+                const uint32_t kb = q / (8 * XT), o = q % (8 * XT);
+                const uint32_t bk = b + kb < a.nbk ? b + kb : a.nbk - 1;
+                p = (const char *) a.xd + ((uint64_t) bk * a.mp + mw) * 4 + o * 16;
+            } else if (q < XS + WS) {
+                const uint32_t qw = q - XS, kb = qw / (4 * WT), o = qw % (4 * WT);
+                const uint32_t bk = b + kb < a.nbk ? b + kb : a.nbk - 1;
+                const uint32_t g0 = nw / 64 + o / 8, g = g0 < a.ng ? g0 : a.ng - 1;
+                p = a.w + a.qbytes + ((uint64_t) g * a.nbk + bk) * 128 + (o % 8) * 16;
+            }
+            if (p) {
+                mmq_dma_v(base + (uint32_t) (QI + wv) * 1024, p);
+            }
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < D - 1; ++s) {
+        if (bb + s * KB < be) {
+            issue(bb + s * KB, s);
+        }
+    }
+    float acc[WM][WN][16];
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                acc[i][j][e] = 0.0f;
+            }
+        }
+    }
+    // The int32 dot comes out as the bits of the float MAGIC + dot (the MFMA adds to
+    // the bits of MAGIC = 1.5 * 2^23, whose ulp is 1; |dot| <= 32 * 128 * 128 < 2^22),
+    // so one subtraction gives float(dot), exactly: with several waves on a SIMD
+    // v_sub_f32 issues at twice the rate of v_cvt_f32_i32 (32 of them: 30 against 54 ns).
+    constexpr float MAGIC = 12582912.0f;
+    mm_i32x16       mg;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        mg[e] = __builtin_bit_cast(int, MAGIC);
+    }
+    const int kg = wv / NP, wp = wv % NP;            // the wave's key group and position
+    const int wm = wp / NN * WM, wn = wp % NN * WN;  // its first tiles
+    // its operands' offsets in a stage (the blocks' own are immediates)
+    const uint32_t xq0 = (uint32_t) (kg * (XT + WT) + wm) * 1024, wq0 = (uint32_t) (kg * (XT + WT) + XT + wn) * 1024;
+    const uint32_t xs0 = (uint32_t) (QI * 1024 + (kg * XT + wm) * 128);
+    const uint32_t ws0 = (uint32_t) (QI * 1024 + XS * 16 + (kg * WT + wn) * 64);
+    auto block = [&](const char * st, int kb) {
+        mm_i32x4 xf[WM], wf[WN];
+        float    sx[WM], sw[WN / 2];
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+            xf[i] = *(const mm_i32x4 *) (st + xq0 + l * 16 + (kb * (XT + WT) + i) * 1024);
+            sx[i] = *(const float *) (st + xs0 + c * 4 + (kb * XT + i) * 128);
+        }
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+            wf[j] = *(const mm_i32x4 *) (st + wq0 + l * 16 + (kb * (XT + WT) + j) * 1024);
+        }
+#pragma unroll
+        for (int j = 0; j < WN / 2; ++j) {
+            sw[j] = (float) *(const _Float16 *) (st + ws0 + l * 2 + (kb * WT + 2 * j) * 64);
+        }
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+#pragma unroll
+            for (int j = 0; j < WN; j += 2) {
+                // the scales d_x[m] d_w[n] of tiles j and j + 1: two 32 x 32 outer products (exact)
+                __builtin_amdgcn_s_setprio(1);
+                const mm_f32x32 sv = __builtin_amdgcn_mfma_f32_32x32x1f32(sx[i], sw[j / 2], mm_f32x32{}, 0, 0, 0);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    __builtin_amdgcn_s_setprio(1);
+                    const mm_i32x16 d = __builtin_amdgcn_mfma_i32_32x32x32_i8(xf[i], wf[j + h], mg, 0, 0, 0);
+                    __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const int bits   = d[e];  // (a copy: a bit cast of the vector element itself takes element 0)
+                        acc[i][j + h][e] =
+                            __builtin_fmaf(__builtin_bit_cast(float, bits) - MAGIC, sv[16 * h + e], acc[i][j + h][e]);
+                    }
+                }
+            }
+        }
+    };
+    uint32_t buf = 0, b = bb;
+    // a stage has landed when its turn comes (each wave waits for its own loads, later
+    // stages' stay in flight), and every wave is done reading the buffer the next loads go to
+    auto next = [&]() {
+        if (b + (D - 2) * KB < be) {
+            if (wv < SCI) {
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((D - 2) * (QI / NW + 1)) : "memory");
+            } else {
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((D - 2) * (QI / NW)) : "memory");
+            }
+        } else {
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+        if (b + (D - 1) * KB < be) {
+            issue(b + (D - 1) * KB, buf == 0 ? D - 1 : buf - 1);
+        }
+    };
+    for (; b + KB <= be; b += KB) {
+        next();
+#pragma unroll
+        for (int kb = 0; kb < KB; kb += KG) {
+            block(lds + buf * STAGE, kb);
+        }
+        buf = buf + 1 == D ? 0 : buf + 1;
+    }
+    if (b < be) {  // the last, partial stage
+        next();
+        for (int kb = 0; b + kb + kg < be; kb += KG) {
+            block(lds + buf * STAGE, kb);
+        }
+    }
+    // Half a tile's outputs per call: D lane l holds column n0 + 32 j + c, rows m0 + 32 i
+    // + 8 q + 4 hh + e (value 4 q + e); v: values e0 .. e0 + 7 of tile (i, j). Row
+    // pointers are uniform (scalar), the lane's part of the address is one offset.
+    const uint32_t m0 = mw + 32 * wm, n0 = nw + 32 * wn;
+    const bool     in  = m0 + 32 * WM <= a.m && n0 + 32 * WN <= a.n;  // uniform: no bounds to check
+    int            el  = l;  // (opaque: nothing of the epilogue's addresses is held over the loop)
+    asm volatile("" : "+v"(el));
+    const int      eh = el >> 5, ec = el & 31;
+    const int64_t  ylo = 4 * eh * a.y1 + 4 * ec, rlo = 4 * eh * a.res1 + 4 * ec;
+    auto store = [&](int i, int j, int e0, float (&v)[8]) {
+        const uint32_t mt0 = m0 + 32 * i + 2 * e0, nt0 = n0 + 32 * j, n = nt0 + ec;
+        if (a.splits > 1) {
+            // the split's sums to the workspace [split][mp][npad] (the rows of the tile lie
+            // inside the padded extent, row groups past the weight are skipped);
+            // k_mmq_reduce adds the splits in order and applies the epilogue
+            if (nt0 < a.npad) {
+                float *        pp = a.part + ((size_t) z * a.mp + mt0) * a.npad + nt0;
+                const uint32_t lo = (uint32_t) (4 * eh) * a.npad + ec;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    (pp + (size_t) (8 * (e / 4) + e % 4) * a.npad)[lo] = v[e];
+                }
+            }
+            return;
+        }
+        if (!in && n >= a.n) {
+            return;
+        }
+        if (a.res != nullptr) {  // the residual values are loaded before any is added
+            const char * rt = a.res + (int64_t) mt0 * a.res1 + (int64_t) nt0 * 4;
+            float        r[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t m = mt0 + 8 * (e / 4) + 4 * eh + e % 4;
+                r[e] = in ? *(const float *) (rt + (int64_t) (8 * (e / 4) + e % 4) * a.res1 + rlo)
+                          : mm_res(a, m < a.m ? m : a.m - 1, n);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[e] = mm_add_res(a, v[e], r[e], n);
+            }
+        }
+        char * yt = a.y + (int64_t) mt0 * a.y1 + (int64_t) nt0 * 4;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (in || mt0 + 8 * (e / 4) + 4 * eh + e % 4 < a.m) {
+                *(float *) (yt + (int64_t) (8 * (e / 4) + e % 4) * a.y1 + ylo) = v[e];
+            }
+        }
+    };
+    // the key groups' sums added in group order, through LDS ([wave][value][lane]);
+    // each group then stores its share of the position's half tiles
+    float * red = (float *) lds;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave is done with the stages
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                red[(wv * WM * WN + i * WN + j) * 1024 + e * 64 + el] = acc[i][j][e];
+            }
+        }
+    }
+    __syncthreads();
+    for (int h = kg; h < 2 * WM * WN; h += KG) {
+        const int t2 = h / 2, e0 = h % 2 * 8;
+        float     v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            v[e] = 0.0f;
+        }
+#pragma unroll
+        for (int g = 0; g < KG; ++g) {
+            const float * rg = red + ((g * NP + wp) * WM * WN + t2) * 1024 + e0 * 64 + el;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[e] = g == 0 ? rg[e * 64] : v[e] + rg[e * 64];
+            }
+        }
+        store(t2 / WN, t2 % WN, e0, v);
+    }
+}
+
 // The matrix kernel's key splits added in split order, then the epilogue
 // (residual, clamp): one thread per output, consecutive threads along a row.
 __global__ void __launch_bounds__(256) k_mmq_reduce(const MmvArgs a) {
@@ -775,6 +1065,9 @@ __global__ void __launch_bounds__(256) k_mmq_reduce(const MmvArgs a) {
     *(float *) (a.y + (int64_t) m * a.y1 + (int64_t) n * 4) = mm_epilogue(a, m, n, t);
 }
 
+#ifndef MI_MMQ64_LONG_BPS
+#define MI_MMQ64_LONG_BPS 96  // blocks per split from which the 64 x 64 tiles split a half-filled grid
+#endif
 #ifndef MI_MMV_NORED_MIN
 #define MI_MMV_NORED_MIN 8  // waves per CU from which key splits stop at one workgroup per row group (0: never)
 #endif
@@ -791,7 +1084,7 @@ void mul_mat_q8_0_plan(MmvArgs & a, int cus) {
     a.qbytes = (uint64_t) a.ng * a.nbk * 2048;
     a.mp     = a.m <= 8 ? a.m : (a.m + 127) / 128 * 128;
     if (a.m > 8) {
-        // the matrix kernel: key splits (workspace partials, added by
+        // the matrix kernels: key splits (workspace partials, added by
         // k_mmq_reduce) only when its 128 x 128 tiles leave resident workgroup
         // slots empty -- the narrow products (n = H) at prefill sizes
         a.wpg             = 1;
@@ -801,6 +1094,23 @@ void mul_mat_q8_0_plan(MmvArgs & a, int cus) {
         ks                = ks > MI_MMQ_MAX_KSPLIT ? MI_MMQ_MAX_KSPLIT : ks;
         ks                = ks > a.nbk / MI_MMQ_MIN_BPS ? a.nbk / MI_MMQ_MIN_BPS : ks;
         ks                = ks < 1 ? 1 : ks;
+        // The 64 x 64 tiles (keys split in the workgroup) while they fit the resident
+        // slots about two and a half times over (512 -> 1152 tiles: 49 against 55 us at 375 x
+        // 12288; 1600: 70 against 64 us at 1537 x 4096), unless a second round of them stands
+        // against 128 x 128 tiles with 3 or 4 key splits (640 tiles, 1024 x 2560 x 4096: 60
+        // against 56 us). Workspace partials on top only where the grid is under a quarter of
+        // the slots (9 x 2048 x 2048: 13.2 with, 16.0 us without; 375 rows: 21.5 and 17.8), or
+        // under half with long key ranges (257 x 2048 x 6144: 29 and 37 us); never more splits
+        // than the 128 x 128 tiles take, so the workspace stays as it was.
+        const uint64_t t64 = (uint64_t) ((a.n + 63) / 64) * ((a.m + 63) / 64);
+        a.tile             = t64 <= sl || (2 * t64 <= 5 * sl && ks < 3) ? 64 : 128;
+        if (a.tile == 64) {
+            const uint64_t k64 = 4 * t64 <= sl ? ks : 2 * t64 <= sl ? a.nbk / MI_MMQ64_LONG_BPS : 1;
+            const uint64_t fit = t64 <= sl ? sl / t64 : 1;
+            ks                 = ks < k64 ? ks : k64;
+            ks                 = ks < fit ? ks : fit;
+            ks                 = ks < 1 ? 1 : ks;
+        }
         a.bps             = a.nbk == 0 ? 1 : (uint32_t) ((a.nbk + ks - 1) / ks);
         a.splits          = a.nbk == 0 ? 1 : (a.nbk + a.bps - 1) / a.bps;
         return;
@@ -888,7 +1198,11 @@ int launch_mul_mat_q8_0(const MmvArgs & a, hipStream_t s) {
         MI_LAUNCH(k_mmv_quant_x, dim3((uint32_t) ((threads + 255) / 256)), dim3(256), 0, s, a);
     }
     if (a.m > 8) {
-        MI_LAUNCH(k_mmq_q8_0, dim3((a.n + 127) / 128, a.mp / 128, a.splits), dim3(256), 0, s, a);
+        if (a.tile == 64) {
+            MI_LAUNCH(k_mmq64_q8_0, dim3((a.n + 63) / 64 * ((a.m + 63) / 64) * a.splits), dim3(512), 0, s, a);
+        } else {
+            MI_LAUNCH(k_mmq_q8_0, dim3((a.n + 127) / 128, a.mp / 128, a.splits), dim3(256), 0, s, a);
+        }
         if (a.splits > 1) {
             const uint64_t outs = (uint64_t) a.m * a.n;
             MI_LAUNCH(k_mmq_reduce, dim3((uint32_t) ((outs + 255) / 256)), dim3(256), 0, s, a);
