@@ -1,0 +1,40 @@
+"""GPU parity of mi_apg_forward where its split over channels and frames changes:
+one or two channels per workgroup (odd channel counts, operands 4-byte aligned
+only), frame counts either side of a workgroup's 512 threads and of the 8192 frames
+held in registers, and out in place of cond. The bar is the op's own: APG runs in
+double and only the order of its sums differs from the oracle's, so the float output
+is within 1 ulp of the oracle's.
+"""
+import numpy as np
+import pytest
+from helpers import to_dev, to_np
+from oracle import oracle as orc
+
+from acestep_ops import sampler as smp
+from acestep_ops.device import DTensor
+
+pytestmark = pytest.mark.gpu
+
+
+def _ulps(y, ref):
+    return np.abs(y.astype(np.float64) - ref) / np.spacing(np.abs(ref).astype(np.float32)).astype(np.float64)
+
+
+@pytest.mark.parametrize("inplace", [False, True])
+@pytest.mark.parametrize("n,t,oc,shift", [(1, 1, 64, 0), (2, 511, 6, 0), (1, 513, 7, 0), (1, 8192, 4, 0), (2, 8193, 2, 0),
+                                          (1, 9300, 3, 0), (1, 6000, 64, 0), (1, 700, 64, 1)])
+def test_apg_frames(dev, n, t, oc, shift, inplace):
+    print(f"apg n={n} t={t} oc={oc} shift={shift} inplace={inplace}", flush=True)
+    r = np.random.default_rng(n + t + oc)
+    ra = np.zeros((n, t, oc))
+    mb = None
+    for step in range(2):
+        cond = r.standard_normal((n, t, oc)).astype(np.float32)
+        unc = (cond - 0.3 * r.standard_normal((n, t, oc))).astype(np.float32)
+        up = lambda a: to_dev(np.concatenate([np.zeros(shift, np.float32), a.ravel()]))[shift:].view(n, t, oc)  # noqa: E731
+        dc, du = up(cond), up(unc)
+        mb = mb if mb is not None else smp.apg_buffer(dc)
+        y = smp.apg_forward(dc, du, 7.0, mb, step == 0, out=dc if inplace else None)
+        y = DTensor(y.buf, (y.buf.nbytes // 4,), "f32").numpy()[-n * t * oc:].reshape(n, t, oc) if inplace else to_np(y)
+        ref = orc.apg_forward(cond, unc, 7.0, ra, step == 0)
+        assert np.max(_ulps(y, ref)) <= 1.0
