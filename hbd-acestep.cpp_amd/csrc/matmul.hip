@@ -529,6 +529,225 @@ __global__ void __launch_bounds__(512) k_mmv_q8_0(const MmvArgs a) {
     }
 }
 
+// Matrix-vector product of one row of x in one launch: the x prologue (the plain
+// quantization, SwiGLU, or [residual add ->] RMSNorm [-> modulate]), the product and
+// the sum of its key splits. At these sizes (one token: 1-25 MB of weights,
+// 4-12 KB of x) a product as prologue, product and split sum is bound by its
+// three launches, each about 3 us with its gap and mostly idle; so every workgroup
+// quantizes all of x itself, from the caches, into LDS, while its first weight blocks
+// are in flight, and holds all key splits of a 64-row group, added in LDS in the order
+// in which k_mmv_q8_0 and k_mmv_reduce add them: the same bits as the three launches. The row's RMS sum is formed the same way in every workgroup (the first
+// one writes the residual sum).
+__global__ void __launch_bounds__(512) k_mmv1_q8_0(const MmvArgs a) {
+    constexpr int          W = 8;  // waves = key splits
+    extern __shared__ char lds[];  // x quants [nbk][32], scales [nbk], the splits' sums [W * splits][64]
+    __shared__ double      rs[W];  // (the first 4 waves sum the squares, in k_mmv_quant_x_norm's order)
+    __shared__ float       scl;
+    const uint32_t g = blockIdx.x;
+    const int      tid = threadIdx.x, l = tid & 63;
+    const int      w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int  T = 64 * W;
+    // the wave's key splits: a.splits in a row of a.bps blocks each
+    const uint32_t bw = a.splits * a.bps;
+    const uint32_t b0 = (uint32_t) w * bw < a.nbk ? (uint32_t) w * bw : a.nbk;
+    const uint32_t b1 = b0 + bw < a.nbk ? b0 + bw : a.nbk;
+    const char *   wq = a.w + (uint64_t) g * a.nbk * 2048 + 16 * l;
+    const char *   wd = a.w + a.qbytes + (uint64_t) g * a.nbk * 128 + 2 * l;
+    constexpr int  U  = MI_MMV_UNROLL;
+    uint4          a0[U], a1[U], c0[U], c1[U];
+    uint16_t       ad[U], cd[U];
+    // a set of U blocks; blocks past the wave's range are clamped to its last one (not used)
+    auto load = [&](uint4 (&w0)[U], uint4 (&w1)[U], uint16_t (&dh)[U], uint32_t bb) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t b = bb + u < b1 ? bb + u : b1 - 1;
+            w0[u]            = ld16(wq + (size_t) b * 2048);
+            w1[u]            = ld16(wq + (size_t) b * 2048 + 1024);
+            dh[u]            = *(const uint16_t *) (wd + (size_t) b * 128);
+        }
+    };
+    if (b0 < b1) {
+        load(a0, a1, ad, b0);
+    }
+    char *  xq = lds;
+    float * xd = (float *) (lds + (size_t) a.nbk * 32);
+    auto    ld4 = [&](const char * p, float (&v)[4]) {
+        if (a.xvec) {
+            const float4 q = *(const float4 *) p;
+            v[0]           = q.x;
+            v[1]           = q.y;
+            v[2]           = q.z;
+            v[3]           = q.w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = ((const float *) p)[e];
+            }
+        }
+    };
+    // x at element i: 4 floats (with the residual sum or the SwiGLU formed)
+    auto xv = [&](uint32_t i, float (&v)[4]) {
+        if (a.glu) {
+            float h[4];
+            ld4(a.g + (int64_t) i * 4, v);
+            ld4(a.u + (int64_t) i * 4, h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = silu_f(v[e]) * h[e];
+            }
+            return;
+        }
+        ld4(a.x + (int64_t) i * 4, v);
+        if (a.ab) {
+            float b4[4];
+            ld4(a.ab + (int64_t) i * 4, b4);
+            if (a.gate) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    b4[e] = b4[e] * a.gate[i + e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = v[e] + b4[e];
+            }
+        }
+    };
+    float scale = 1.0f;
+    if (a.nw) {
+        double ss = 0.0;
+        for (uint32_t i = tid < 256 ? 4u * (uint32_t) tid : a.k; i < a.k; i += 1024u) {
+            float v[4];
+            xv(i, v);
+            if (a.sum && g == 0) {
+                float * sp = (float *) a.sum + i;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sp[e] = v[e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                ss += (double) (v[e] * v[e]);
+            }
+        }
+        ss = group_sum<64>(ss);
+        if (l == 0) {
+            rs[w] = ss;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            scl = rms_scale(rs[0] + rs[1] + rs[2] + rs[3], (int) a.k, a.eps);
+        }
+        __syncthreads();
+        scale = scl;
+    }
+    const uint32_t sub = (uint32_t) tid & 7u;
+    for (uint32_t b = (uint32_t) tid >> 3; b < a.nbk; b += (uint32_t) T / 8) {  // the 8 lanes of a block share b
+        const uint32_t i0 = b * 32u + sub * 4u;
+        float          f[4];
+        xv(i0, f);
+        if (a.nw) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v = f[e] * scale;
+                f[e]          = v * a.nw[i0 + e];
+            }
+            if (a.msc) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    f[e] = f[e] * (a.msc[i0 + e] + 1.0f);
+                    f[e] = f[e] + a.msh[i0 + e];
+                }
+            }
+        }
+        float amax = fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fmaxf(fabsf(f[2]), fabsf(f[3])));
+        amax       = group_max<8>(amax);
+        const float d  = mm_div127(amax);
+        const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
+        uint32_t    qv = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float q = __builtin_amdgcn_fmed3f(__builtin_rintf(f[e] * id), -128.0f, 127.0f);
+            qv |= ((uint32_t) (int32_t) q & 0xffu) << (8 * e);
+        }
+        *(uint32_t *) (xq + (size_t) b * 32 + sub * 4) = qv;
+        if (sub == 0) {
+            xd[b] = (float) __builtin_bit_cast(_Float16, f32_to_f16_bits(d));
+        }
+    }
+    __syncthreads();
+    float    acc  = 0.0f;
+    float *  red  = xd + a.nbk;  // [split][lane]
+    uint32_t vs   = (uint32_t) w * a.splits, left = a.bps;  // the split, its blocks left
+    for (uint32_t q = 0; q < a.splits; ++q) {
+        red[(vs + q) * 64 + l] = 0.0f;
+    }
+    // a set's dots, straight-line: the LDS reads of all its blocks are in flight together
+    // (a block past the range reads the last one and adds 0 * dot)
+    auto run = [&](const uint4 (&w0)[U], const uint4 (&w1)[U], const uint16_t (&dh)[U], uint32_t bb) {
+        uint4 x0[U], x1[U];
+        float xs[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t b  = bb + u < b1 ? bb + u : b1 - 1;
+            const uint4 *  xb = (const uint4 *) (xq + (size_t) b * 32);
+            x0[u]             = xb[0];
+            x1[u]             = xb[1];
+            xs[u]             = xd[b];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t wv[8] = { w0[u].x, w0[u].y, w0[u].z, w0[u].w, w1[u].x, w1[u].y, w1[u].z, w1[u].w };
+            const uint32_t xw[8] = { x0[u].x, x0[u].y, x0[u].z, x0[u].w, x1[u].x, x1[u].y, x1[u].z, x1[u].w };
+            int            isum  = 0;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                isum = __builtin_amdgcn_sdot4((int) wv[q], (int) xw[q], isum, false);
+            }
+            const float dw = (float) __builtin_bit_cast(_Float16, dh[u]);
+            const float v  = __builtin_fmaf((float) isum, dw * xs[u], acc);
+            acc            = bb + u < b1 ? v : acc;
+            if (--left == 0 || bb + u + 1 == b1) {  // uniform: the split's last block
+                if (bb + u < b1) {
+                    red[vs * 64 + l] = acc;
+                }
+                acc  = 0.0f;
+                left = a.bps;
+                ++vs;
+            }
+        }
+    };
+    // two register sets of U blocks: one's loads are in flight while the other's dots run
+    for (uint32_t b = b0; b < b1; b += 2 * U) {
+        if (b + U < b1) {
+            load(c0, c1, cd, b + U);
+        }
+        run(a0, a1, ad, b);
+        if (b + 2 * U < b1) {
+            load(a0, a1, ad, b + 2 * U);
+        }
+        if (b + U < b1) {
+            run(c0, c1, cd, b + U);
+        }
+    }
+    const uint32_t row = g * 64 + l;
+    __syncthreads();
+    if (w == 0 && row < a.n) {
+        // the splits of a workgroup of k_mmv_q8_0 in wave order, those sums in k_mmv_reduce's
+        float v = 0.0f;
+        for (uint32_t s1 = 0; s1 < a.splits; ++s1) {
+            float p = 0.0f;
+#pragma unroll
+            for (uint32_t w2 = 0; w2 < (uint32_t) W; ++w2) {
+                p += w2 < a.wpg ? red[(s1 * a.wpg + w2) * 64 + l] : 0.0f;
+            }
+            v += p;
+        }
+        *(float *) (a.y + (int64_t) row * 4) = mm_epilogue(a, 0, row, v);
+    }
+}
+
 // y[m][row] = sum over the workgroups' partials, in workgroup order (splits > 1)
 template <int M>
 __global__ void __launch_bounds__(256) k_mmv_reduce(const MmvArgs a) {
@@ -1115,6 +1334,13 @@ void mul_mat_q8_0_plan(MmvArgs & a, int cus) {
         a.splits          = a.nbk == 0 ? 1 : (a.nbk + a.bps - 1) / a.bps;
         return;
     }
+    // One row of x in one launch where a wave's share of the keys is at most one set of 4
+    // blocks, or two sets on a grid whose weights want the whole chip anyway (us, this and
+    // the three launches: 1024 -> 6144 6.7 and 7.6, 2048 -> 12288 10.9 and 11.9; the
+    // others with the waves' sums added without the splits' order, about 1 us quicker: 2048
+    // -> 2048 7.5 and 7.1, 2560 -> 6144 9.9 and 9.9, 6144 -> 2048 15.6 and 9.0). Past 512 row
+    // groups the prologue repeated in each outweighs it (1024 -> 151669 with the norm: 38 and 27).
+    a.one = a.m == 1 && a.nbk > 0 && a.ng <= 512 && (a.nbk <= 32 || (a.nbk <= 64 && a.ng >= 128));
     const uint32_t want = (uint32_t) (cus > 0 ? cus : 256) * MI_MMV_WAVES_PER_CU;
     uint32_t       s    = a.ng == 0 || a.ng >= want ? 1 : (want + a.ng - 1) / a.ng;
     // when one workgroup per row group (its splits added in LDS) still gives the
@@ -1180,8 +1406,27 @@ static void launch_quant_x_norm8(const MmvArgs & a, hipStream_t s) {
     }
 }
 
+// Whether y shares memory with an operand that every workgroup of the one-launch kernel
+// reads (or with the residual sum): then the product waits for the prologue's own launch.
+static bool mmv1_overlaps(const MmvArgs & a) {
+    const uintptr_t y0 = (uintptr_t) a.y, y1 = y0 + (uintptr_t) a.n * 4;
+    for (const void * p : { (const void *) a.x, (const void *) a.ab, (const void *) a.g, (const void *) a.u,
+                            (const void *) a.sum, (const void *) a.nw, (const void *) a.gate, (const void *) a.msc,
+                            (const void *) a.msh }) {
+        const uintptr_t q = (uintptr_t) p;
+        if (p != nullptr && q < y1 && y0 < q + (uintptr_t) a.k * 4) {
+            return true;
+        }
+    }
+    return false;
+}
+
 int launch_mul_mat_q8_0(const MmvArgs & a, hipStream_t s) {
     if (a.n == 0 || a.m == 0) {
+        return MI_OK;
+    }
+    if (a.one && !mmv1_overlaps(a)) {
+        MI_LAUNCH(k_mmv1_q8_0, dim3(a.ng), dim3(512), (size_t) a.nbk * 36 + (size_t) a.splits * 8 * 256, s, a);
         return MI_OK;
     }
     if (a.nw && a.m >= (uint32_t) MI_QXN8_MIN_ROWS && a.nbk <= 4 * 32) {

@@ -1,0 +1,60 @@
+"""GPU parity of mi_mul_mat_q8_0 on one row of x, where the prologue, the product and
+the key sum are one launch (up to 32 blocks of keys, or 64 on 128 or more row groups):
+the oracle's bar at ragged and smallest sizes and either side of the rule, each
+prologue equal to its separate op followed by the plain product, and y sharing memory
+with an input (which keeps the separate launches).
+"""
+import numpy as np
+import pytest
+from helpers import assert_mul_mat_q8_0, to_dev, to_np
+from oracle import oracle as orc
+
+from acestep_ops import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(n, k, seed):
+    r = np.random.default_rng(seed)
+    w = orc.quantize_q8_0(r.standard_normal((n, k)).astype(np.float32))
+    return r, w, r.standard_normal((1, k)).astype(np.float32), ops.q8_0_repack(ops.Q8(to_dev(w)))
+
+
+@pytest.mark.parametrize("n,k", [(1, 32), (64, 64), (65, 288), (130, 992), (1024, 1024), (32768, 96), (32769, 96), (300, 1056),
+                                 (8128, 2048), (8129, 2016), (8192, 2048), (8192, 2080)])
+def test_sizes(dev, n, k):
+    print(f"mul_mat q8_0 one row n={n} k={k}", flush=True)
+    r, w, x, wr = _case(n, k, n + k)
+    assert_mul_mat_q8_0(to_np(ops.mul_mat_q8_0(wr, to_dev(x))), w, x)
+    x[:] = 0.0
+    assert not to_np(ops.mul_mat_q8_0(wr, to_dev(x))).any()
+
+
+@pytest.mark.parametrize("n,k,shift", [(130, 1024, 0), (200, 96, 1), (8200, 2048, 0)])
+def test_prologues(dev, n, k, shift):
+    """shift 1: operands 4-byte aligned only."""
+    print(f"mul_mat q8_0 one row prologues n={n} k={k} shift={shift}", flush=True)
+    r, w, x, wr = _case(n, k, n + k)
+    up = lambda a: to_dev(np.concatenate([np.zeros(shift, np.float32), a.ravel()]))[shift:].view(*a.shape)  # noqa: E731
+    f = lambda *s: r.standard_normal(s).astype(np.float32)  # noqa: E731
+    dx, b, g, nw, sc, sh = up(x), up(f(1, k)), to_dev(f(k)), to_dev(f(k)), to_dev(f(k)), to_dev(f(k))
+    gu, res = up(f(1, 2 * k)), to_dev(f(1, n))
+    eq = lambda y, z: np.testing.assert_array_equal(to_np(y), to_np(z))  # noqa: E731
+    eq(ops.mul_mat_q8_0_rms_norm(wr, dx, nw, 1e-6), ops.mul_mat_q8_0(wr, ops.rms_norm(dx, 1e-6, w=nw)))
+    eq(ops.mul_mat_q8_0_swiglu_add(wr, gu, res), ops.add(ops.mul_mat_q8_0(wr, ops.swiglu(gu)), res))
+    s, y = ops.mul_mat_q8_0_add_rms_norm(wr, dx, b, nw, 1e-6)
+    s2, n2 = ops.add_rms_norm(dx, b, 1e-6, w=nw)
+    eq(s, s2)
+    eq(y, ops.mul_mat_q8_0(wr, n2))
+    s, y = ops.mul_mat_q8_0_adaln(wr, dx, nw, 1e-6, b=b, gate=g, scale=sc, shift=sh)
+    s2, n2 = ops.add_rms_norm(dx, b, 1e-6, gate=g, w=nw, scale=sc, shift=sh)
+    eq(s, s2)
+    eq(y, ops.mul_mat_q8_0(wr, n2))
+
+
+def test_y_in_place_of_x(dev):
+    print("mul_mat q8_0 one row in place", flush=True)
+    _, w, x, wr = _case(1024, 1024, 5)
+    dx = to_dev(x)
+    ops.mul_mat_q8_0(wr, dx, out=dx)
+    assert_mul_mat_q8_0(to_np(dx), w, x)
