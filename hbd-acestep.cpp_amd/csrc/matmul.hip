@@ -733,16 +733,21 @@ __global__ void __launch_bounds__(512) k_mmv1_q8_0(const MmvArgs a) {
     }
     const uint32_t row = g * 64 + l;
     __syncthreads();
+    // the splits of a workgroup of k_mmv_q8_0 in wave order, a wave each, and then those
+    // sums in k_mmv_reduce's order
+    for (uint32_t s1 = (uint32_t) w; s1 < a.splits; s1 += (uint32_t) W) {
+        float p = 0.0f;
+#pragma unroll
+        for (uint32_t w2 = 0; w2 < (uint32_t) W; ++w2) {
+            p += w2 < a.wpg ? red[(s1 * a.wpg + w2) * 64 + l] : 0.0f;
+        }
+        red[s1 * a.wpg * 64 + l] = p;  // (this wave's own lane read it)
+    }
+    __syncthreads();
     if (w == 0 && row < a.n) {
-        // the splits of a workgroup of k_mmv_q8_0 in wave order, those sums in k_mmv_reduce's
         float v = 0.0f;
         for (uint32_t s1 = 0; s1 < a.splits; ++s1) {
-            float p = 0.0f;
-#pragma unroll
-            for (uint32_t w2 = 0; w2 < (uint32_t) W; ++w2) {
-                p += w2 < a.wpg ? red[(s1 * a.wpg + w2) * 64 + l] : 0.0f;
-            }
-            v += p;
+            v += red[s1 * a.wpg * 64 + l];
         }
         *(float *) (a.y + (int64_t) row * 4) = mm_epilogue(a, 0, row, v);
     }
@@ -1336,7 +1341,7 @@ void mul_mat_q8_0_plan(MmvArgs & a, int cus) {
     }
     // One row of x in one launch where a wave's share of the keys is at most one set of 4
     // blocks, or two sets on a grid whose weights want the whole chip anyway (us, this and
-    // the three launches: 1024 -> 6144 6.7 and 7.6, 2048 -> 12288 10.9 and 11.9; the
+    // the three launches: 1024 -> 6144 6.4 and 7.6, 2048 -> 12288 10.7 and 11.9; the
     // others with the waves' sums added without the splits' order, about 1 us quicker: 2048
     // -> 2048 7.5 and 7.1, 2560 -> 6144 9.9 and 9.9, 6144 -> 2048 15.6 and 9.0). Past 512 row
     // groups the prologue repeated in each outweighs it (1024 -> 151669 with the norm: 38 and 27).
