@@ -1411,19 +1411,22 @@ static void launch_quant_x_norm8(const MmvArgs & a, hipStream_t s) {
     }
 }
 
-// Whether y shares memory with an operand that every workgroup of the one-launch kernel
-// reads (or with the residual sum): then the product waits for the prologue's own launch.
+// Whether a workgroup of the one-launch kernel would write what another still reads: y, or
+// the residual sum (the entry point refuses it over its addends only), sharing memory with
+// an operand that every workgroup reads, or with each other. Then the prologue keeps its
+// own launch, whose one workgroup has read the operands in its order before y is written.
 static bool mmv1_overlaps(const MmvArgs & a) {
-    const uintptr_t y0 = (uintptr_t) a.y, y1 = y0 + (uintptr_t) a.n * 4;
-    for (const void * p : { (const void *) a.x, (const void *) a.ab, (const void *) a.g, (const void *) a.u,
-                            (const void *) a.sum, (const void *) a.nw, (const void *) a.gate, (const void *) a.msc,
-                            (const void *) a.msh }) {
-        const uintptr_t q = (uintptr_t) p;
-        if (p != nullptr && q < y1 && y0 < q + (uintptr_t) a.k * 4) {
+    const uintptr_t kb = (uintptr_t) a.k * 4;
+    auto over = [&](const void * p, uintptr_t bytes, const void * q) {  // q: k floats
+        return p != nullptr && q != nullptr && (uintptr_t) q < (uintptr_t) p + bytes && (uintptr_t) p < (uintptr_t) q + kb;
+    };
+    for (const void * q : { (const void *) a.x, (const void *) a.ab, (const void *) a.g, (const void *) a.u,
+                            (const void *) a.nw, (const void *) a.gate, (const void *) a.msc, (const void *) a.msh }) {
+        if (over(a.y, (uintptr_t) a.n * 4, q) || over(a.sum, kb, q)) {
             return true;
         }
     }
-    return false;
+    return over(a.y, (uintptr_t) a.n * 4, a.sum);
 }
 
 int launch_mul_mat_q8_0(const MmvArgs & a, hipStream_t s) {

@@ -58,3 +58,20 @@ def test_y_in_place_of_x(dev):
     dx = to_dev(x)
     ops.mul_mat_q8_0(wr, dx, out=dx)
     assert_mul_mat_q8_0(to_np(dx), w, x)
+
+
+@pytest.mark.parametrize("over", ["norm", "shift"])
+def test_sum_over_a_vector(dev, over):
+    """The residual sum written over the norm weight or the modulate's shift, which every row's
+    norm reads after it: the bits of the sum first, then the product with the sum in their place."""
+    print(f"mul_mat q8_0 one row, sum over {over}", flush=True)
+    n, k = 6144, 1024
+    r, _, x, wr = _case(n, k, 11)
+    f = lambda *s: r.standard_normal(s).astype(np.float32)  # noqa: E731
+    dx, b, nw, sc, sh = to_dev(x), to_dev(f(1, k)), to_dev(f(k)), to_dev(f(k)), to_dev(f(k))
+    s0 = ops.add(dx, b)
+    nw2, sh2 = (s0.view(k), sh) if over == "norm" else (nw, s0.view(k))
+    ref = ops.mul_mat_q8_0(wr, ops.add_rms_norm(dx, b, 1e-6, w=nw2, scale=sc, shift=sh2)[1])
+    s, y = ops.mul_mat_q8_0_adaln(wr, dx, nw, 1e-6, b=b, scale=sc, shift=sh, out_sum=(nw if over == "norm" else sh).view(1, k))
+    np.testing.assert_array_equal(to_np(s), to_np(s0))
+    np.testing.assert_array_equal(to_np(y), to_np(ref))
