@@ -539,10 +539,11 @@ __global__ void __launch_bounds__(512) k_mmv_q8_0(const MmvArgs a) {
 // in which k_mmv_q8_0 and k_mmv_reduce add them: the same bits as the three launches. The row's RMS sum is formed the same way in every workgroup (the first
 // one writes the residual sum).
 __global__ void __launch_bounds__(512) k_mmv1_q8_0(const MmvArgs a) {
-    constexpr int          W = 8;  // waves = key splits
-    extern __shared__ char lds[];  // x quants [nbk][32], scales [nbk], the splits' sums [W * splits][64]
-    __shared__ double      rs[W];  // (the first 4 waves sum the squares, in k_mmv_quant_x_norm's order)
-    __shared__ float       scl;
+    constexpr int W = 8;  // waves = key splits
+    // x quants [nbk][32], read 16 bytes at a time, scales [nbk], the splits' sums [W * splits][64]
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    __shared__ double rs[W];  // (the first 4 waves sum the squares, in k_mmv_quant_x_norm's order)
+    __shared__ float  scl;
     const uint32_t g = blockIdx.x;
     const int      tid = threadIdx.x, l = tid & 63;
     const int      w = __builtin_amdgcn_readfirstlane(tid >> 6);
