@@ -1349,7 +1349,7 @@ int mi_apg_forward(const mi_tensor * cond, const mi_tensor * uncond, float guida
         return MI_ERR_PARAM;
     }
     if (cond->ne[0] > 1024) {
-        return MI_ERR_UNSUPPORTED;  // channels per workgroup
+        return MI_ERR_UNSUPPORTED;  // a sample's workgroup has a thread per channel
     }
     const size_t need = (size_t) nelements(*cond) * sizeof(double);
     if (need > 0 && (!momentum_buf || momentum_bytes < need)) {

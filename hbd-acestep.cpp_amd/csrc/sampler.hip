@@ -10,9 +10,9 @@
 //                          inv = 1 / |cond_c| (0 if |cond_c|^2 <= 1e-60)
 //                          dot = sum_t (s ra) (cond inv)
 //   out = (float) (cond + (scale - 1) (s ra - dot cond inv))
-// One workgroup per one or two channels of a sample, threads split the frames; the
-// three per-channel sums (|ra|^2, |cond|^2, ra . cond) reduce in LDS, then a
-// second pass writes the result. Layout [N][T][Oc] (ggml [Oc, T, N]).
+// One workgroup per one or two channels of a sample, or per sample where there are
+// many; threads split the frames; the three per-channel sums (|ra|^2, |cond|^2,
+// ra . cond) reduce in LDS, then a second pass writes the result. Layout [N][T][Oc] (ggml [Oc, T, N]).
 //
 // Solvers (solvers/solver-euler.h, solver-dpm.h) and the final step
 // (dit-sampler.h:601-605), in fp32 with the reference's operation order:
@@ -22,8 +22,67 @@
 //   final:  out = xt - vt * t
 #include "common.h"
 #include "launch.h"
+#include "rules.h"
 
 namespace mi {
+
+// One workgroup per sample, for many samples (rules.h): lanes own channels, waves split
+// the frames, every line is read whole. With samples enough to fill the chip it runs at
+// HBM rate (256 x 1500 frames of 64 channels: 227 us, 4.3 TB/s of what it moves); a few
+// samples leave it a chain of loads per thread (2 x 6000: 502 us against 41 below).
+__global__ void __launch_bounds__(1024) k_apg_sample(const ApgArgs a) {
+    extern __shared__ double red[];  // [3][nph][oc], then [3][oc]
+    const uint32_t b   = blockIdx.x;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t oc = a.oc, nph = blockDim.x / a.oc;
+    const uint32_t c = tid % oc, ph = tid / oc;  // blockDim is nph * oc: every thread has a (channel, phase)
+    const float * cond = a.cond + (size_t) b * a.t * oc;
+    const float * unc  = a.uncond + (size_t) b * a.t * oc;
+    double *      ra   = a.ra + (size_t) b * a.t * oc;
+    float *       out  = a.out + (size_t) b * a.t * oc;
+    double        s_rr = 0.0, s_cc = 0.0, s_rc = 0.0;
+    for (uint32_t t = ph; t < a.t; t += nph) {
+        const size_t i  = (size_t) t * oc + c;
+        const double cv = (double) cond[i];
+        const double d  = cv - (double) unc[i];
+        const double r  = a.first ? d : d + a.momentum * ra[i];
+        ra[i]           = r;
+        s_rr += r * r;
+        s_cc += cv * cv;
+        s_rc += r * cv;
+    }
+    red[(0 * nph + ph) * oc + c] = s_rr;
+    red[(1 * nph + ph) * oc + c] = s_cc;
+    red[(2 * nph + ph) * oc + c] = s_rc;
+    __syncthreads();
+    double * fin = red + 3 * nph * oc;  // per channel: s, inv, dot
+    if (ph == 0) {
+        double rr = 0.0, cc = 0.0, rc = 0.0;
+        for (uint32_t p = 0; p < nph; ++p) {
+            rr += red[(0 * nph + p) * oc + c];
+            cc += red[(1 * nph + p) * oc + c];
+            rc += red[(2 * nph + p) * oc + c];
+        }
+        const double norm = sqrt(rr > 0.0 ? rr : 0.0);
+        double       s    = 1.0;
+        if (a.threshold > 0.0f && norm > 1e-60) {
+            s = fmin(1.0, (double) a.threshold / norm);
+        }
+        const double inv = cc > 1e-60 ? 1.0 / sqrt(cc) : 0.0;
+        fin[c]           = s;
+        fin[oc + c]      = inv;
+        fin[2 * oc + c]  = s * inv * rc;
+    }
+    __syncthreads();
+    const double s = fin[c], inv = fin[oc + c], dot = fin[2 * oc + c];
+    const double w = (double) a.scale - 1.0;
+    for (uint32_t t = ph; t < a.t; t += nph) {
+        const size_t i    = (size_t) t * oc + c;
+        const double cv   = (double) cond[i];
+        const double orth = s * ra[i] - dot * (cv * inv);
+        out[i]            = (float) (cv + w * orth);
+    }
+}
 
 // One workgroup per CG channels of a sample: the sums run over a channel's frames
 // only, so the channels spread over the chip without partial sums in memory. What
@@ -428,8 +487,12 @@ int launch_apg(const ApgArgs & a, hipStream_t s) {
         return MI_OK;
     }
     // two channels per workgroup where the rows' alignment allows 8- and 16-byte accesses
-    const uintptr_t f = (uintptr_t) a.cond | (uintptr_t) a.uncond | (uintptr_t) a.out;
-    if (a.oc % 2 == 0 && f % 8 == 0 && (uintptr_t) a.ra % 16 == 0) {
+    const uintptr_t f  = (uintptr_t) a.cond | (uintptr_t) a.uncond | (uintptr_t) a.out;
+    const uint32_t  cg = a.oc % 2 == 0 && f % 8 == 0 && (uintptr_t) a.ra % 16 == 0 ? 2 : 1;
+    if (apg_by_sample(a.n, a.t, a.oc, cg)) {
+        const uint32_t nph = 1024 / a.oc;
+        MI_LAUNCH(k_apg_sample, dim3(a.n), dim3(nph * a.oc), (size_t) (3 * nph * a.oc + 3 * a.oc) * sizeof(double), s, a);
+    } else if (cg == 2) {
         MI_LAUNCH(k_apg<2>, dim3(a.oc / 2, a.n), dim3(APG_T), 0, s, a);
     } else {
         MI_LAUNCH(k_apg<1>, dim3(a.oc, a.n), dim3(APG_T), 0, s, a);

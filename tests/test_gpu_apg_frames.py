@@ -38,3 +38,20 @@ def test_apg_frames(dev, n, t, oc, shift, inplace):
         y = DTensor(y.buf, (y.buf.nbytes // 4,), "f32").numpy()[-n * t * oc:].reshape(n, t, oc) if inplace else to_np(y)
         ref = orc.apg_forward(cond, unc, 7.0, ra, step == 0)
         assert np.max(_ulps(y, ref)) <= 1.0
+
+
+@pytest.mark.parametrize("n,t,oc", [(1, 31, 64), (40, 17, 64), (200, 40, 7), (3, 2, 1024), (130, 300, 64), (66000, 1, 2)])
+def test_apg_many_samples(dev, n, t, oc):
+    """A workgroup per sample: short ones, many, one frame more than the workgroup's phases, and
+    more samples than a grid's second dimension holds."""
+    print(f"apg by sample n={n} t={t} oc={oc}", flush=True)
+    r = np.random.default_rng(n + t + oc)
+    ra = np.zeros((n, t, oc))
+    mb = None
+    for step in range(2):
+        cond = r.standard_normal((n, t, oc)).astype(np.float32)
+        unc = (cond - 0.3 * r.standard_normal((n, t, oc))).astype(np.float32)
+        dc, du = to_dev(cond), to_dev(unc)
+        mb = mb if mb is not None else smp.apg_buffer(dc)
+        y = to_np(smp.apg_forward(dc, du, 7.0, mb, step == 0))
+        assert np.max(_ulps(y, orc.apg_forward(cond, unc, 7.0, ra, step == 0))) <= 1.0

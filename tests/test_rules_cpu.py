@@ -1,0 +1,33 @@
+"""The dispatch rules of csrc/rules.h at sizes where both sides were timed on the card:
+the quicker side is taken (sizes within 5 % of each other are left to the rule).
+"""
+import os
+import subprocess
+
+from helpers import ROOT
+
+APG = [  # n, t, oc, channels per workgroup, us by sample, us by channels
+    (1, 6000, 64, 2, 482.1, 38.8), (2, 6000, 64, 2, 502.1, 41.0), (4, 1500, 64, 2, 113.9, 14.1), (4, 375, 64, 2, 22.0, 5.9),
+    (1, 100, 64, 2, 7.7, 4.3), (1, 12, 64, 2, 3.3, 4.2), (8, 4, 64, 2, 3.1, 4.6), (32, 100, 64, 2, 8.4, 14.5),
+    (32, 750, 64, 2, 63.5, 36.5), (128, 375, 64, 2, 39.1, 87.2), (128, 750, 64, 2, 76.9, 130.9), (64, 6000, 64, 2, 641.7, 405.4),
+    (256, 6000, 64, 2, 902.6, 1662.4), (512, 25, 64, 2, 7.2, 196.9), (512, 1500, 64, 2, 396.3, 868.9),
+    (256, 750, 8, 2, 17.4, 39.9), (64, 12, 8, 2, 6.4, 4.7), (1, 750, 8, 2, 10.2, 5.0),
+    (256, 750, 7, 1, 16.8, 52.1), (256, 3000, 7, 1, 47.3, 170.9), (8, 200, 7, 1, 8.1, 3.9), (256, 3000, 1, 1, 39.2, 9.0),
+    (1, 750, 1024, 2, 964.0, 18.2), (16, 750, 1024, 2, 1050.0, 265.1), (8, 12, 1024, 2, 12.8, 50.5), (256, 25, 1024, 2, 53.7, 1551.7),
+]
+
+
+def _run(tmp_path, expr, rows):
+    src = tmp_path / "r.cpp"
+    body = "".join(f"    printf(\"%d\\n\", (int) ({expr(r)}));\n" for r in rows)
+    src.write_text('#include "rules.h"\n#include <cstdio>\nusing namespace mi;\nint main() {\n' + body + "}\n")
+    exe = tmp_path / "r"
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "hbd-acestep.cpp_amd", "csrc"), str(src), "-o", str(exe)],
+                   check=True)
+    return [int(v) for v in subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split()]
+
+
+def test_apg_takes_the_quicker_split(tmp_path):
+    got = _run(tmp_path, lambda r: f"apg_by_sample({r[0]}, {r[1]}, {r[2]}, {r[3]})", APG)
+    bad = [r for r, g in zip(APG, got) if g != (r[4] < r[5])]
+    assert not bad, bad
