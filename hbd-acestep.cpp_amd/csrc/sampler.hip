@@ -489,7 +489,11 @@ int launch_apg(const ApgArgs & a, hipStream_t s) {
     // two channels per workgroup where the rows' alignment allows 8- and 16-byte accesses
     const uintptr_t f  = (uintptr_t) a.cond | (uintptr_t) a.uncond | (uintptr_t) a.out;
     const uint32_t  cg = a.oc % 2 == 0 && f % 8 == 0 && (uintptr_t) a.ra % 16 == 0 ? 2 : 1;
-    if (apg_by_sample(a.n, a.t, a.oc, cg)) {
+    // out laid over uncond, but not in place of it: another channel's workgroup may still
+    // read what one writes; a sample's one workgroup has read all of uncond before
+    const uintptr_t o = (uintptr_t) a.out, u = (uintptr_t) a.uncond, bytes = (uintptr_t) a.n * a.t * a.oc * 4;
+    const bool      over = o != u && o < u + bytes && u < o + bytes;
+    if (over || apg_by_sample(a.n, a.t, a.oc, cg)) {
         const uint32_t nph = 1024 / a.oc;
         MI_LAUNCH(k_apg_sample, dim3(a.n), dim3(nph * a.oc), (size_t) (3 * nph * a.oc + 3 * a.oc) * sizeof(double), s, a);
     } else if (cg == 2) {

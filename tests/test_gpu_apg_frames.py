@@ -55,3 +55,22 @@ def test_apg_many_samples(dev, n, t, oc):
         mb = mb if mb is not None else smp.apg_buffer(dc)
         y = to_np(smp.apg_forward(dc, du, 7.0, mb, step == 0))
         assert np.max(_ulps(y, orc.apg_forward(cond, unc, 7.0, ra, step == 0))) <= 1.0
+
+
+@pytest.mark.parametrize("by", [1, -1, 3])
+def test_apg_out_across_uncond(dev, by):
+    """out of one sample laid over uncond, frames later or earlier."""
+    print(f"apg out across uncond by={by}", flush=True)
+    t, oc = 1200, 64
+    r = np.random.default_rng(50 + by)
+    cond = r.standard_normal((1, t, oc)).astype(np.float32)
+    unc = (cond - 0.3 * r.standard_normal((1, t, oc))).astype(np.float32)
+    whole = np.zeros(((t + 4) * oc,), np.float32)
+    at, to = (0, by) if by > 0 else (-by, 0)
+    whole[at * oc:(at + t) * oc] = unc.ravel()
+    d = to_dev(whole)
+    dc = to_dev(cond)
+    v = lambda f: d[f * oc:(f + t) * oc].view(1, t, oc)  # noqa: E731
+    smp.apg_forward(dc, v(at), 7.0, smp.apg_buffer(dc), True, out=v(to))
+    y = to_np(d)[to * oc:(to + t) * oc].reshape(1, t, oc)
+    assert np.max(_ulps(y, orc.apg_forward(cond, unc, 7.0, np.zeros((1, t, oc)), True))) <= 1.0
