@@ -192,7 +192,7 @@ struct MmvArgs {
     int64_t      y1;
     uint32_t     splits, wpg, bps;  // workgroups per row group, waves (key splits) per workgroup,
                                     // blocks per wave (set by mul_mat_q8_0_plan)
-    uint32_t     one;     // 1: 1 or 2 rows of x, everything in one launch
+    uint32_t     one;     // 1: one row of x, everything in one launch
     uint32_t     tile;    // the matrix kernel's workgroup tile, 128 or 64 rows of x and of w
     const float * nw;          // non-null: x = rms_norm(x) * nw (the norm prologue), with eps
     float        eps;

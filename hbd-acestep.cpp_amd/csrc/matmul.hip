@@ -22,6 +22,7 @@
 // adds them in workgroup order, so the result does not depend on scheduling.
 #include "common.h"
 #include "launch.h"
+#include "rules.h"
 
 namespace mi {
 
@@ -1340,13 +1341,6 @@ void mul_mat_q8_0_plan(MmvArgs & a, int cus) {
         a.splits          = a.nbk == 0 ? 1 : (a.nbk + a.bps - 1) / a.bps;
         return;
     }
-    // One row of x in one launch where a wave's share of the keys is at most one set of 4
-    // blocks, or two sets on a grid whose weights want the whole chip anyway (us, this and
-    // the three launches: 1024 -> 6144 6.4 and 7.6, 2048 -> 12288 10.7 and 11.9; the
-    // others with the waves' sums added without the splits' order, about 1 us quicker: 2048
-    // -> 2048 7.5 and 7.1, 2560 -> 6144 9.9 and 9.9, 6144 -> 2048 15.6 and 9.0). Past 512 row
-    // groups the prologue repeated in each outweighs it (1024 -> 151669 with the norm: 38 and 27).
-    a.one = a.m == 1 && a.nbk > 0 && a.ng <= 512 && (a.nbk <= 32 || (a.nbk <= 64 && a.ng >= 128));
     const uint32_t want = (uint32_t) (cus > 0 ? cus : 256) * MI_MMV_WAVES_PER_CU;
     uint32_t       s    = a.ng == 0 || a.ng >= want ? 1 : (want + a.ng - 1) / a.ng;
     // when one workgroup per row group (its splits added in LDS) still gives the
@@ -1363,6 +1357,7 @@ void mul_mat_q8_0_plan(MmvArgs & a, int cus) {
     a.wpg    = s < 8 ? s : 8;
     a.splits = (s + a.wpg - 1) / a.wpg;                       // workgroups per row group
     a.bps    = a.nbk == 0 ? 1 : (a.nbk + a.splits * a.wpg - 1) / (a.splits * a.wpg);
+    a.one    = a.m == 1 && a.nbk > 0 && mmv_one_launch(a.nbk, a.ng);
 }
 
 static size_t al256(size_t v) {

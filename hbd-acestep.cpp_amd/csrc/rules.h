@@ -6,6 +6,25 @@
 
 namespace mi {
 
+// Q8_0 product of one row of x (nbk key blocks, ng groups of 64 weight rows): whether the
+// prologue, the product and the key sum are one launch of a workgroup per row group. A
+// wave takes an eighth of the keys (up to a block per split more), in sets of 4 blocks.
+// us with the norm prologue, three launches / one, weights of 400 MB in turn:
+//   1024 keys: 64 groups 8.0 / 5.6, 96 8.3 / 5.7, 256 7.4 / 6.5, 512 10.0 / 9.3, 2370 29.8 / 35.0
+//   2048 keys: 96 groups 11.0 / 8.4, 192 13.4 / 9.5, 512 16.1 / 14.4; 6144 keys: 32 groups 12.0 / 14.2
+// Past 256 row groups the product has no second sum to save, and a second round of
+// workgroups stands against one: there it wins only with the sets near full (32 and 64
+// blocks 0.93, 24 0.99, 48 0.99; 8 blocks 1.11, 16 1.03, 33 1.07, 40 1.07). Up to 128 row
+// groups 33-80 blocks would win too (64 blocks 32 groups 7.8 / 7.2, 80 blocks 96 groups
+// 11.5 / 9.2; 96 blocks 16 groups 8.9 / 9.3) but keep the three launches.
+inline bool mmv_one_launch(uint32_t nbk, uint32_t ng) {
+    if (ng > 512 || nbk > 64 || (nbk > 32 && ng < 128)) {
+        return false;
+    }
+    const uint32_t share = (nbk + 7) / 8, sets = (share + 3) / 4;
+    return ng <= 256 || share >= sets * 3;  // at most a quarter of the sets' slots empty
+}
+
 // APG: whether a workgroup takes a whole sample (its frames in rows of oc channels)
 // instead of one or two channels of it (cg). The channel split fills the chip where
 // there are few samples, but each of its workgroups takes a line request per frame for

@@ -1,5 +1,6 @@
 """GPU parity of mi_mul_mat_q8_0 on one row of x, where the prologue, the product and
-the key sum are one launch (up to 32 blocks of keys, or 64 on 128 or more row groups):
+the key sum are one launch (up to 32 blocks of keys, or 64 on 128 or more row groups; past
+256 row groups where the waves' sets of blocks are nearly full):
 the oracle's bar at ragged and smallest sizes and either side of the rule, each
 prologue equal to its separate op followed by the plain product, and y sharing memory
 with an input (which keeps the separate launches).
@@ -21,7 +22,8 @@ def _case(n, k, seed):
 
 
 @pytest.mark.parametrize("n,k", [(1, 32), (64, 64), (65, 288), (130, 992), (1024, 1024), (32768, 96), (32769, 96), (300, 1056),
-                                 (8128, 2048), (8129, 2016), (8192, 2048), (8192, 2080)])
+                                 (8128, 2048), (8129, 2016), (8192, 2048), (8192, 2080),
+                                 (16384, 256), (16385, 256), (16385, 768), (16385, 1056)])
 def test_sizes(dev, n, k):
     print(f"mul_mat q8_0 one row n={n} k={k}", flush=True)
     r, w, x, wr = _case(n, k, n + k)

@@ -16,6 +16,13 @@ APG = [  # n, t, oc, channels per workgroup, us by sample, us by channels
     (1, 750, 1024, 2, 964.0, 18.2), (16, 750, 1024, 2, 1050.0, 265.1), (8, 12, 1024, 2, 12.8, 50.5), (256, 25, 1024, 2, 53.7, 1551.7),
 ]
 
+ONE_ROW = [  # key blocks, groups of 64 weight rows, us in three launches, us in one (norm prologue)
+    (32, 16, 7.2, 5.3), (32, 64, 8.0, 5.6), (32, 96, 8.3, 5.7), (32, 204, 10.0, 7.3), (32, 256, 7.4, 6.5), (32, 320, 8.8, 8.3),
+    (32, 512, 10.0, 9.3), (64, 192, 13.4, 9.6), (64, 256, 11.0, 9.7), (64, 320, 13.1, 12.1), (64, 512, 16.1, 14.4),
+    (33, 128, 9.3, 6.7), (33, 288, 9.4, 9.9), (40, 320, 9.5, 10.3), (8, 288, 5.4, 6.2), (8, 512, 5.9, 6.6), (16, 288, 6.4, 6.8),
+    (192, 32, 12.0, 14.2), (32, 2370, 29.8, 35.0),
+]
+
 
 def _run(tmp_path, expr, rows):
     src = tmp_path / "r.cpp"
@@ -30,4 +37,10 @@ def _run(tmp_path, expr, rows):
 def test_apg_takes_the_quicker_split(tmp_path):
     got = _run(tmp_path, lambda r: f"apg_by_sample({r[0]}, {r[1]}, {r[2]}, {r[3]})", APG)
     bad = [r for r, g in zip(APG, got) if g != (r[4] < r[5])]
+    assert not bad, bad
+
+
+def test_one_row_takes_the_quicker_route(tmp_path):
+    got = _run(tmp_path, lambda r: f"mmv_one_launch({r[0]}, {r[1]})", ONE_ROW)
+    bad = [r for r, g in zip(ONE_ROW, got) if g != (r[3] < r[2])]
     assert not bad, bad
