@@ -1320,16 +1320,13 @@ void mul_mat_q8_0_plan(MmvArgs & a, int cus) {
         ks                = ks > MI_MMQ_MAX_KSPLIT ? MI_MMQ_MAX_KSPLIT : ks;
         ks                = ks > a.nbk / MI_MMQ_MIN_BPS ? a.nbk / MI_MMQ_MIN_BPS : ks;
         ks                = ks < 1 ? 1 : ks;
-        // The 64 x 64 tiles (keys split in the workgroup) while they fit the resident
-        // slots about two and a half times over (512 -> 1152 tiles: 49 against 55 us at 375 x
-        // 12288; 1600: 70 against 64 us at 1537 x 4096), unless a second round of them stands
-        // against 128 x 128 tiles with 3 or 4 key splits (640 tiles, 1024 x 2560 x 4096: 60
-        // against 56 us). Workspace partials on top only where the grid is under a quarter of
-        // the slots (9 x 2048 x 2048: 13.2 with, 16.0 us without; 375 rows: 21.5 and 17.8), or
-        // under half with long key ranges (257 x 2048 x 6144: 29 and 37 us); never more splits
-        // than the 128 x 128 tiles take, so the workspace stays as it was.
+        // With the 64 x 64 tiles (keys split in the workgroup) workspace partials on top only
+        // where the grid is under a quarter of the slots (9 x 2048 x 2048: 13.2 with, 16.0 us
+        // without; 375 rows: 21.5 and 17.8), or under half with long key ranges (257 x 2048 x
+        // 6144: 29 and 37 us); never more splits than the 128 x 128 tiles take, so the
+        // workspace stays as it was.
         const uint64_t t64 = (uint64_t) ((a.n + 63) / 64) * ((a.m + 63) / 64);
-        a.tile             = t64 <= sl || (2 * t64 <= 5 * sl && ks < 3) ? 64 : 128;
+        a.tile             = mmq_small_tiles(t64, sl, ks, a.nbk) ? 64 : 128;
         if (a.tile == 64) {
             const uint64_t k64 = 4 * t64 <= sl ? ks : 2 * t64 <= sl ? a.nbk / MI_MMQ64_LONG_BPS : 1;
             const uint64_t fit = t64 <= sl ? sl / t64 : 1;

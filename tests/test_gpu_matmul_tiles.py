@@ -42,9 +42,9 @@ def test_small_tile_key_splits(dev, n, k, m):
     assert np.array_equal(y, to_np(ops.mul_mat_q8_0(wr, to_dev(x))))  # the same bits on every call
 
 
-@pytest.mark.parametrize("n,k,m", [(12288, 64, 700), (8200, 160, 1100), (2560, 3072, 1024)])
+@pytest.mark.parametrize("n,k,m", [(12288, 64, 700), (8200, 160, 1100), (2560, 3072, 1024), (2560, 6144, 1217), (2100, 96, 1000)])
 def test_large_tile(dev, n, k, m):
-    """Grids past the 64 x 64 tiles' share, the last with 3 key splits."""
+    """Grids past the 64 x 64 tiles' share, with 3 and 2 key splits and with short keys."""
     print(f"mul_mat q8_0 128-tile n={n} k={k} m={m}", flush=True)
     _, w, x, wr = _case(n, k, m, n + k + m)
     assert_mul_mat_q8_0(to_np(ops.mul_mat_q8_0(wr, to_dev(x))), w, x)

@@ -23,6 +23,14 @@ ONE_ROW = [  # key blocks, groups of 64 weight rows, us in three launches, us in
     (192, 32, 12.0, 14.2), (32, 2370, 29.8, 35.0),
 ]
 
+TILES = [  # 64 x 64 tiles, resident workgroups, key splits of the 128 x 128 tiles, key blocks, us 128 x 128, us 64 x 64 (or per cent)
+    (1, 512, 4, 64, 27.5, 13.2), (288, 512, 4, 64, 54.8, 49.3), (512, 512, 2, 64, 31.9, 21.4), (512, 512, 4, 304, 100.0, 90.0),
+    (1152, 512, 1, 64, 54.8, 49.3), (1600, 512, 1, 64, 64.0, 70.0), (640, 512, 3, 128, 56.0, 60.0), (800, 512, 2, 304, 131.6, 134.4),
+    (672, 512, 2, 192, 100.0, 89.0), (770, 512, 2, 192, 93.5, 84.7), (1024, 512, 2, 192, 100.0, 94.0), (1088, 512, 1, 20, 100.0, 94.0), (960, 512, 1, 12, 100.0, 93.0),
+    (640, 512, 1, 8, 100.0, 92.0), (768, 512, 1, 8, 100.0, 92.0), (768, 512, 1, 5, 100.0, 104.0), (1088, 512, 1, 8, 100.0, 107.0), (1078, 512, 1, 5, 100.0, 122.0), (544, 512, 1, 1, 100.0, 110.0),
+    (912, 512, 1, 4, 14.4, 15.2), (1088, 512, 1, 1, 100.0, 131.0),
+]
+
 
 def _run(tmp_path, expr, rows):
     src = tmp_path / "r.cpp"
@@ -43,4 +51,10 @@ def test_apg_takes_the_quicker_split(tmp_path):
 def test_one_row_takes_the_quicker_route(tmp_path):
     got = _run(tmp_path, lambda r: f"mmv_one_launch({r[0]}, {r[1]})", ONE_ROW)
     bad = [r for r, g in zip(ONE_ROW, got) if g != (r[3] < r[2])]
+    assert not bad, bad
+
+
+def test_products_take_the_quicker_tiles(tmp_path):
+    got = _run(tmp_path, lambda r: f"mmq_small_tiles({r[0]}, {r[1]}, {r[2]}, {r[3]})", TILES)
+    bad = [r for r, g in zip(TILES, got) if g != (r[5] < r[4])]
     assert not bad, bad
