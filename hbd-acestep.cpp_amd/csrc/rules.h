@@ -32,8 +32,9 @@ inline bool mmv_one_launch(uint32_t nbk, uint32_t ng) {
 // is the one exception found). Past that, up to two and a half times over (us, 128 / 64):
 //   one round of 128 x 128 tiles, 64 key blocks: 1152 tiles 55 / 49, 1600 tiles 64 / 70
 //   3 or 4 key splits stand against their second round: 640 tiles, 128 blocks 56 / 60
-//   2 key splits, long keys: 800 tiles, 304 blocks 132 / 134; of the time 0.89-0.94 at 768
-//     and 770 tiles, 0.94 at 1024; 128 blocks and shorter 0.95
+//   2 key splits: 0.85-0.95 of the time, at 800 tiles of 192 blocks or more 1.00-1.02 (304
+//     blocks, 1217 rows 132 / 134; the 64 x 64 tiles all the same: they need no partials, and
+//     the call without a workspace of its own takes sizes that partials would not leave room for)
 //   short keys: the pipeline's start and the sum of the key groups weigh more the more tiles
 //     a CU gets in turn: of the time, with 3 tiles per CU (768) 8 blocks 0.92, 6 1.0, 5 1.04,
 //     1 1.11; with 4 (1024) 12 blocks 0.93, 10 1.0, 5 1.13; with 5 (1280) 16 blocks 0.97, 12 1.0,
@@ -42,11 +43,8 @@ inline bool mmq_small_tiles(uint64_t t64, uint64_t slots, uint64_t ks, uint32_t 
     if (t64 <= slots) {
         return true;
     }
-    if (ks >= 3 || (ks == 2 && nbk >= 192 && 20 * t64 > 31 * slots && 4 * t64 <= 7 * slots)) {
-        return false;
-    }
     const uint64_t cu = (2 * t64 + slots - 1) / slots;  // tiles per CU
-    return cu <= 5 && nbk >= 4 * (cu - 1);
+    return ks < 3 && cu <= 5 && nbk >= 4 * (cu - 1);
 }
 
 // APG: whether a workgroup takes a whole sample (its frames in rows of oc channels)

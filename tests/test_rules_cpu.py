@@ -25,7 +25,7 @@ ONE_ROW = [  # key blocks, groups of 64 weight rows, us in three launches, us in
 
 TILES = [  # 64 x 64 tiles, resident workgroups, key splits of the 128 x 128 tiles, key blocks, us 128 x 128, us 64 x 64 (or per cent)
     (1, 512, 4, 64, 27.5, 13.2), (288, 512, 4, 64, 54.8, 49.3), (512, 512, 2, 64, 31.9, 21.4), (512, 512, 4, 304, 100.0, 90.0),
-    (1152, 512, 1, 64, 54.8, 49.3), (1600, 512, 1, 64, 64.0, 70.0), (640, 512, 3, 128, 56.0, 60.0), (800, 512, 2, 304, 131.6, 134.4),
+    (1152, 512, 1, 64, 54.8, 49.3), (1600, 512, 1, 64, 64.0, 70.0), (640, 512, 3, 128, 56.0, 60.0),
     (672, 512, 2, 192, 100.0, 89.0), (770, 512, 2, 192, 93.5, 84.7), (1024, 512, 2, 192, 100.0, 94.0), (1088, 512, 1, 20, 100.0, 94.0), (960, 512, 1, 12, 100.0, 93.0),
     (640, 512, 1, 8, 100.0, 92.0), (768, 512, 1, 8, 100.0, 92.0), (768, 512, 1, 5, 100.0, 104.0), (1088, 512, 1, 8, 100.0, 107.0), (1078, 512, 1, 5, 100.0, 122.0), (544, 512, 1, 1, 100.0, 110.0),
     (912, 512, 1, 4, 14.4, 15.2), (1088, 512, 1, 1, 100.0, 131.0),
