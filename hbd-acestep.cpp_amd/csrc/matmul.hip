@@ -994,18 +994,13 @@ __global__ void __launch_bounds__(256) k_mmq_q8_0(const MmvArgs a) {
 // 54.8 -> 49.3, 1537 rows of 2048 -> 2048 45.9 -> 42.9. On large grids it loses
 // (12288 x 1024 rows: 110 against 89): twice the operand traffic per output.
 
-// 16 bytes per lane from base + off straight into LDS at dst + 16 * lane (dst uniform)
+// 16 bytes per lane from base + off straight into LDS at dst + 16 * lane (dst uniform; the
+// instruction takes it from m0, which the compiler sets, a wait state before)
 __device__ __forceinline__ void mmq_dma(uint32_t dst, const char * base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(dst), "v"(off), "s"(base)
-                 : "memory", "m0");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "{m0}"(dst), "v"(off), "s"(base) : "memory");
 }
 __device__ __forceinline__ void mmq_dma_v(uint32_t dst, const char * p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                 :
-                 : "s"(dst), "v"(p)
-                 : "memory", "m0");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "{m0}"(dst), "v"(p) : "memory");
 }
 
 __global__ void __launch_bounds__(512, 4) k_mmq64_q8_0(const MmvArgs a) {
