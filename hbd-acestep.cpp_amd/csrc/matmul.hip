@@ -982,11 +982,11 @@ __global__ void __launch_bounds__(256) k_mmq_q8_0(const MmvArgs a) {
 // rows of x x 64 weight rows each) x 4 key groups: every stage of 4 blocks gives each
 // key group one, and the groups' sums are added in group order in LDS, so the keys
 // are split over 4 waves without partials in memory or a second launch. What bounds
-// it is the latency of one wave's chain of blocks (an LDS read, two MFMAs, 64
-// conversions and fmas), so the split is over keys and the operands are fetched ahead:
+// it is the latency of one wave's chain of blocks (LDS reads, 3 MFMAs, 32 subtractions
+// and 32 fmas), so the split is over keys and the operands are fetched ahead:
 // global_load_lds copies them into LDS 3 stages (12 blocks) before use, in MFMA lane
-// order, so that the reads are linear and conflict-free; up to 128 VGPRs keep 4 waves
-// per SIMD (2 workgroups per CU). The block's scales are two f32 outer products by one
+// order, so that the reads are linear and conflict-free; 124 VGPRs without a spill keep
+// 4 waves per SIMD (2 workgroups per CU). The block's scales are two f32 outer products by one
 // v_mfma_f32_32x32x1_2b (K = 1: a lane holds one d_x and one d_w, no zero slots to
 // build). Measured against the 128 x 128 kernel (x quantization and split sum
 // included, us, 2048 -> 2048 / 2048 -> 12288): 9 rows 27.5 ->
@@ -1170,8 +1170,8 @@ __global__ void __launch_bounds__(512, 4) k_mmq64_q8_0(const MmvArgs a) {
         }
         buf = buf + 1 == D ? 0 : buf + 1;
     }
-    if (b < be) {  // the last, partial stage
-        next();
+    if (b < be) {  // the last, partial stage: nothing is left to issue
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         for (int kb = 0; b + kb + kg < be; kb += KG) {
             block(lds + buf * STAGE, kb);
         }
