@@ -62,6 +62,43 @@ def test_y_in_place_of_x(dev):
     assert_mul_mat_q8_0(to_np(dx), w, x)
 
 
+@pytest.mark.parametrize("bad", [False, True])
+@pytest.mark.parametrize("n,k", [(1024, 1024), (6144, 1024), (130, 992), (65, 32), (10944, 992), (12288, 2048), (8200, 1056)])
+def test_same_bits_as_separate_launches(dev, n, k, bad):
+    """y sharing memory with an operand keeps the separate launches: the bits of the one launch,
+    for each prologue and each operand that is checked (12288 x 2048: 3 splits of 3 blocks per
+    wave, the last with one block; bad: NaN and infinite elements of x)."""
+    print(f"mul_mat q8_0 one row, bits n={n} k={k} bad={bad}", flush=True)
+    r, _, x, wr = _case(n, k, n + k)
+    f = lambda *s: r.standard_normal(s).astype(np.float32)  # noqa: E731
+    b, gu, nw, sc, sh, g = f(1, k), f(1, 2 * k), f(k), f(k), f(k), f(k)
+    if bad:
+        x[0, [3, 17]], gu[0, [5, k + 9]] = (np.nan, np.inf), (-np.inf, np.nan)
+
+    def over(a):
+        """(a on the device, y over its first n elements)"""
+        d = to_dev(np.concatenate([a.ravel(), np.zeros(max(n - a.size, 0), np.float32)]))
+        return d[:a.size].view(*a.shape), d[:n].view(1, n)
+
+    eq = lambda y, z: np.testing.assert_array_equal(to_np(y), to_np(z))  # noqa: E731
+    dx, y = over(x)
+    eq(ops.mul_mat_q8_0(wr, dx, out=y), ops.mul_mat_q8_0(wr, to_dev(x)))
+    dg, y = over(gu)
+    eq(ops.mul_mat_q8_0_swiglu(wr, dg, out=y), ops.mul_mat_q8_0_swiglu(wr, to_dev(gu)))
+    ops_ = {"x": x, "b": b, "nw": nw, "sc": sc, "sh": sh, "g": g}
+    call = lambda d, **kw: ops.mul_mat_q8_0_adaln(  # noqa: E731
+        wr, d["x"], d["nw"], 1e-6, b=d["b"], gate=d["g"], scale=d["sc"], shift=d["sh"], **kw)
+    s0, y0 = call({q: to_dev(v) for q, v in ops_.items()})
+    for name in ops_:
+        d = {q: to_dev(v) for q, v in ops_.items() if q != name}
+        d[name], y = over(ops_[name])
+        s1, y1 = call(d, out=y)
+        eq(s1, s0)
+        eq(y1, y0)
+    sm, y = over(np.zeros_like(x))  # y over the sum: the product comes last
+    eq(call({q: to_dev(v) for q, v in ops_.items()}, out=y, out_sum=sm)[1], y0)
+
+
 @pytest.mark.parametrize("over", ["norm", "shift"])
 def test_sum_over_a_vector(dev, over):
     """The residual sum written over the norm weight or the modulate's shift, which every row's
