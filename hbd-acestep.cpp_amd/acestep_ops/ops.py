@@ -409,7 +409,7 @@ def mul_mat_q8_0_adaln(w: Q8R64, a, norm_w, eps: float, b=None, gate=None, scale
 
 
 def mul_mat_q8_0(w: Q8R64, x, out=None, workspace=None, stream=None):
-    """ggml_mul_mat(w, x): x F32 (m, k) with m <= 8 -> F32 (m, n)."""
+    """ggml_mul_mat(w, x): x F32 (m, k) -> F32 (m, n)."""
     y = _out(out, tuple(x.shape[:-1]) + (w.n,), "f32")
     need = mul_mat_q8_0_workspace(w, x)
     ws = workspace

@@ -19,7 +19,13 @@
 // across the wave and read through the scalar cache; sdot4 per 4 quants. Up to
 // 8 key splits of a row group share a workgroup and are added in LDS in wave
 // order; with more, each workgroup writes its partial sums and a small kernel
-// adds them in workgroup order, so the result does not depend on scheduling.
+// adds them in workgroup order, so the result does not depend on scheduling. One row
+// of x can run as one launch instead of the quantization, the product and that sum.
+//
+// Matrix kernels (more than 8 rows): int8 MFMAs for the block dots, the scales applied
+// to every block. 128 x 128 outputs per workgroup with operands from global memory and,
+// on idle grids, key splits through memory; or 64 x 64 with the keys split over four wave
+// groups of the workgroup and operands through LDS. rules.h says which call takes which.
 #include "common.h"
 #include "launch.h"
 #include "rules.h"
@@ -537,8 +543,10 @@ __global__ void __launch_bounds__(512) k_mmv_q8_0(const MmvArgs a) {
 // three launches, each about 3 us with its gap and mostly idle; so every workgroup
 // quantizes all of x itself, from the caches, into LDS, while its first weight blocks
 // are in flight, and holds all key splits of a 64-row group, added in LDS in the order
-// in which k_mmv_q8_0 and k_mmv_reduce add them: the same bits as the three launches. The row's RMS sum is formed the same way in every workgroup (the first
-// one writes the residual sum).
+// in which k_mmv_q8_0 and k_mmv_reduce add them: the same bits as the three launches. A
+// wave's share is its splits times a.bps blocks: up to 8, or 9 (3 sets, the last of one
+// block) with 3 splits of 3 blocks at 171 to 204 row groups. The row's RMS sum is formed
+// the same way in every workgroup (the first one writes the residual sum).
 __global__ void __launch_bounds__(512) k_mmv1_q8_0(const MmvArgs a) {
     constexpr int W = 8;  // waves = key splits
     // x quants [nbk][32], read 16 bytes at a time, scales [nbk], the splits' sums [W * splits][64]
@@ -686,7 +694,7 @@ __global__ void __launch_bounds__(512) k_mmv1_q8_0(const MmvArgs a) {
         red[(vs + q) * 64 + l] = 0.0f;
     }
     // a set's dots, straight-line: the LDS reads of all its blocks are in flight together
-    // (a block past the range reads the last one and adds 0 * dot)
+    // (a block past the range reads the last one, its dot is dropped by a select)
     auto run = [&](const uint4 (&w0)[U], const uint4 (&w1)[U], const uint16_t (&dh)[U], uint32_t bb) {
         uint4 x0[U], x1[U];
         float xs[U];
