@@ -545,7 +545,7 @@ __global__ void __launch_bounds__(512) k_mmv_q8_0(const MmvArgs a) {
 // are in flight, and holds all key splits of a 64-row group, added in LDS in the order
 // in which k_mmv_q8_0 and k_mmv_reduce add them: the same bits as the three launches. A
 // wave's share is its splits times a.bps blocks: up to 8, or 9 (3 sets, the last of one
-// block) with 3 splits of 3 blocks at 171 to 204 row groups. The row's RMS sum is formed
+// block) with 3 splits of 3 blocks at 171 to 255 row groups. The row's RMS sum is formed
 // the same way in every workgroup (the first one writes the residual sum).
 __global__ void __launch_bounds__(512) k_mmv1_q8_0(const MmvArgs a) {
     constexpr int W = 8;  // waves = key splits
