@@ -30,7 +30,9 @@ inline bool mmv_one_launch(uint32_t nbk, uint32_t ng) {
 // key splits; slots = resident workgroups. While they fit the slots they win everywhere
 // measured (9 rows to 512 tiles; 592 weight rows x 498 blocks x 1625 rows 123 against 118 us
 // is the one exception found). Past that, up to two and a half times over (us, 128 / 64):
-//   one round of 128 x 128 tiles, 64 key blocks: 1152 tiles 55 / 49, 1600 tiles 64 / 70
+//   64 key blocks: 1152 tiles 55 / 49, 1600 64 / 70; past 5 tiles per CU the times cross back
+//     and forth (64-80 blocks: of the time, 1344-1536 tiles 0.88-0.97, 2016 0.91-0.94, 2432
+//     1.08, 3344 0.93) and the 128 x 128 tiles stay
 //   3 or 4 key splits stand against their second round: 640 tiles, 128 blocks 56 / 60
 //   2 key splits: 0.85-0.95 of the time, at 800 tiles of 192 blocks or more 1.00-1.02 (304
 //     blocks, 1217 rows 132 / 134; the 64 x 64 tiles all the same: they need no partials, and
